@@ -233,6 +233,51 @@ def run(s):
     return s["out"]
 
 
+def exact(case, seed):
+    """What `run` returns for these inputs in float64: the dense weights, no rounding between the layers of a chain.  The
+    inputs are drawn in the order in which `prepare` draws them.  An encoding is whole numbers and has none."""
+    if case["kind"] == "encode":
+        return None
+    gen = torch.Generator(device=DEVICE)
+    gen.manual_seed(seed)
+
+    def weight(M, K):
+        return _weight(gen, M, K, case["sparsity"], case["pruning"])
+
+    def bias(M):
+        return (torch.rand(M, generator=gen, device=DEVICE) - 0.5).half().double()
+
+    def product(x, W, b, act):
+        y = x @ W.double().t()
+        if b is not None:
+            y += b
+        if act == S.ACT_RELU:
+            y = y.relu()
+        elif act == S.ACT_GELU:
+            y = torch.nn.functional.gelu(y, approximate="tanh")
+        return y
+
+    if case["kind"] == "linear":
+        W = weight(case["M"], case["K"])
+        x = _activations(gen, case["N"], case["K"]).double()
+        return product(x, W, bias(case["M"]) if case["bias"] else None, case["act"])
+    D, F, N = case["D"], case["F"], case["N"]
+    outs, h = [], _activations(gen, N, D).double()
+    for _ in range(case["layers"]):
+        linears = []
+        for M, K, act in ((3 * D, D, S.ACT_NONE), (D, D, S.ACT_NONE), (F, D, S.ACT_RELU), (D, F, S.ACT_NONE)):
+            W = weight(M, K)
+            linears.append((W, bias(M), act))
+        attended = _activations(gen, N, D).double()
+        qkv, proj, ffn1, ffn2 = linears
+        a = product(h, *qkv)
+        b = product(attended, *proj)
+        c = product(b, *ffn1)
+        h = product(c, *ffn2)
+        outs += [a, b, c, h]
+    return outs
+
+
 def _weight_bytes(M, K, sparsity):
     """Compressed arrays of one matrix: fp16 values, one 64-bit bitmap per 8x8 tile, one offset per group tile."""
     return 2 * (1 - sparsity) * M * K + M * K / 8 + 4 * (M * K // 4096 + 1)
