@@ -221,7 +221,8 @@ int SpMM_EncodeDevice_Values(hipStream_t stream, const void* W, int M, int K, co
  *                    irrelevant on entry (the call clears it).  After the call has finished, scratch's second
  *                    32-bit word is 0 on success; bit 1 (value 2) says `values` was too small (bitmaps and offsets
  *                    are complete, some runs were not written), bit 0 that a workgroup gave up waiting for its
- *                    predecessors (nothing is valid then; not expected on a healthy device).
+ *                    predecessors (nothing is valid then; not expected on a healthy device).  Unless bit 0 is
+ *                    set, the third word is offsets[G]: one 16-byte copy brings the status and the count.
  * Asynchronous on `stream`; returns the launch status, or 1 for M or K not a multiple of 64 or a missing or
  * misaligned scratch.  No counterpart in the reference.
  */

@@ -262,7 +262,7 @@ constexpr int      kStage = 2048;
 constexpr int      kOnePassWaves = 16; // waves = group tiles per chunk: what one ticket buys
 
 struct OnePassHeader {
-    unsigned ticket, error, pad0, pad1;
+    unsigned ticket, error, count, pad; // count: offsets[G], beside the error word so that one copy brings both
 };
 
 __global__ __launch_bounds__(256) void zero_words(unsigned* p, size_t n)
@@ -429,6 +429,8 @@ __global__ __launch_bounds__(64 * kOnePassWaves, 8) void encode_onepass(
         offsets[g + 1] = (int)(base + (unsigned)padded);
         if (g == 0)
             offsets[0] = 0;
+        if (g == G - 1)
+            head->count = (unsigned)(base + (unsigned)padded);
     }
     if (base + (unsigned)padded > capacity) {
         if (lane == 0)
