@@ -744,6 +744,39 @@ def test_bias_activation_entry_point(torch, oracle, M, K, N, s, sk, act, with_bi
         assert np.array_equal(C.view(np.uint16), dev.spmm(X, sk).view(np.uint16))
 
 
+@pytest.mark.parametrize("M,K,N", [(256, 64, 64), (320, 192, 128), (512, 640, 384)])
+@pytest.mark.parametrize("act", [0, 1, 2])
+@pytest.mark.parametrize("with_bias", [False, True])
+def test_unsplit_tail_of_the_wide_kernel_equals_the_reduction(torch, variants_lib, M, K, N, act, with_bias):
+    """At Split_K = 1 the wide kernel applies bias and activation to its accumulators, the row-per-lane kernel leaves
+    them to the reduction.  With exact sums (small integers) both round the same fp32 value once: equal bit for bit."""
+    import ctypes as C
+    rng = np.random.default_rng(M + N)
+    W, X = _small_integer_problem(rng, M, K, N, 0.5)
+    dev = Device(torch, S.InitSparseMatrixA_bitmap(W))
+    x = torch.from_numpy(X.view(np.int16).copy()).to("cuda:0")
+    bias = rng.uniform(-2, 2, M).astype(np.float16)
+    bias[[0, 63, M - 1]] = [np.inf, -np.inf, -0.0]
+    b = torch.from_numpy(bias.view(np.int16).copy()).to("cuda:0") if with_bias else None
+    call = variants_lib.SpMM_SplitK_API_BiasAct
+    call.restype, call.argtypes = C.c_int, [C.c_void_p] * 6 + [C.c_int] * 3 + [C.c_void_p, C.c_int, C.c_void_p, C.c_int]
+    got = []
+    try:
+        for variant in (3, 4):
+            print(f"case tail M={M} K={K} N={N} act={act} bias={with_bias} variant={variant}", flush=True)
+            variants_lib.SpMM_Debug_SetKernelVariant(variant)
+            out = torch.full((N, M), 0x7e00, dtype=torch.int16, device="cuda:0")
+            ws = torch.empty(4 * M * N, dtype=torch.uint8, device="cuda:0")
+            assert call(torch.cuda.current_stream().cuda_stream, dev.values.data_ptr(), dev.bitmaps.data_ptr(),
+                        dev.offsets.data_ptr(), x.data_ptr(), out.data_ptr(), M, N, K, ws.data_ptr(), 1,
+                        b.data_ptr() if with_bias else None, act) == 0
+            torch.cuda.synchronize()
+            got.append(out.cpu().numpy())
+    finally:
+        variants_lib.SpMM_Debug_SetKernelVariant(2)
+    assert np.array_equal(got[0], got[1])
+
+
 def test_bias_activation_errors_and_layer(torch, oracle, capfd):
     t = torch.zeros(64, dtype=torch.int16, device="cuda:0")
     assert S.SpMM_SplitK_API_BiasAct(None, t, t, t, t, t, 64, 16, 64, t, 1, None, 7) == S.api.HIP_ERROR_INVALID_VALUE
