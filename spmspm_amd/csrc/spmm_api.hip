@@ -76,7 +76,21 @@ int auto_split_k_wide(int M, int N, int K)
 //   partials a split adds the reduction kernel, and every batch writes and re-reads an fp32 slab of M*N.
 int auto_split_k(int M, int N, int K)
 {
-    if (spmm::use_wide_kernel(M, N, K))
+    if (spmm::kernel_by_split(M, N, K)) { // split and kernel together
+        int    best   = 1;
+        double best_c = 1e30;
+        for (int sk = 1; sk <= 32 && sk <= K / 64; ++sk) {
+            const double c = (spmm::use_wide_kernel(M, N, K, sk) ? spmm::main_wide_us(M, N, K, sk)
+                                                                 : spmm::main_rows_us(M, N, K, sk)) +
+                             spmm::split_us(M, N, sk);
+            if (c < best_c - 1e-9) {
+                best_c = c;
+                best   = sk;
+            }
+        }
+        return best;
+    }
+    if (spmm::use_wide_kernel(M, N, K, 1))
         return auto_split_k_wide(M, N, K);
     const int    nkb  = K / 64;
     const long   base = (long)(M / 64) * spmm::column_blocks(N);
@@ -646,7 +660,7 @@ extern "C" const char* SpMM_KernelName(int M, int N, int K, int Split_K)
     thread_local char name[64];
     const int         sk   = Split_K <= 0 ? split_k_for(M, N, K) : clamp_split_k(Split_K, K);
     const char*       fp32 = sk > 1 ? "true" : "false"; // SpMM_SplitK_API: partial sums in fp32 whenever K is split
-    if (spmm::use_wide_kernel(M, N, K))
+    if (spmm::use_wide_kernel(M, N, K, sk))
         std::snprintf(name, sizeof name, "spmm::spmm_bitmap_wide<%d, %s>", spmm::wide_tile_n(N) / 16, fp32);
     else
         std::snprintf(name, sizeof name, "spmm::spmm_bitmap_rows<%d, %s>", spmm::tile_n(N) / 16, fp32);

@@ -2,6 +2,8 @@
 import os
 import re
 
+import pytest
+
 import spmspm_amd as S
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -270,6 +272,25 @@ def test_kernel_name_follows_the_dispatch():
     assert name(9216, 24, 36864, 1) == "" and name(100, 16, 64, 1) == ""
     # the name is that of SpMM_SplitK_API / _Sized / _NoAlloc: fp32 partial sums exactly when K is split
     assert name(5120, 16, 5120, 1).endswith("false>") and name(5120, 16, 5120, 2).endswith("true>")
+
+
+@pytest.mark.parametrize("M,N,K,splits", [
+    (5120, 2048, 5120, {0: "wide<8", 1: "wide<8", 4: "wide<8"}),   # fills the chip many times over: wide at any split
+    (4160, 384, 4928, {0: "wide<8", 2: "rows<4", 5: "wide<8"}),    # 102 workgroups at Split_K 2, 255 at 5
+    (2048, 1024, 2048, {0: "rows<4", 1: "rows<4"}),                # one full round of rows, a quarter of one of wide
+    (192, 2048, 8192, {0: "rows<4", 1: "rows<4"}),                 # fewer than 256 rows
+    (9216, 256, 64, {0: "rows<4", 1: "rows<4"}),                   # one k block
+])
+def test_kernel_of_a_small_matrix_with_many_columns_follows_its_split(M, N, K, splits):
+    """From N = 256 on the kernel depends on the split of the call.  The library's own split stays within what it can
+    use, its workspace is that of the split it names, and the entry point without workspace names one that fits."""
+    for sk, kernel in splits.items():
+        assert kernel in S.library().SpMM_KernelName(M, N, K, sk).decode(), (sk, kernel)
+    auto = S.SpMM_SplitK_Auto(M, N, K)
+    assert 1 <= auto <= min(32, K // 64)
+    assert S.SpMM_WorkspaceBytes(M, N, K, 0) == (4 * M * N * auto if auto > 1 else 0)
+    own = S.SpMM_SplitK_AutoNoAlloc(M, N, K)
+    assert own == 1 or 4 * M * N * own <= S.api.NOALLOC_SCRATCH_BYTES
 
 
 def test_row_count_limit_is_reported(capfd):
