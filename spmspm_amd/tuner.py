@@ -31,7 +31,9 @@ def candidate_splits(K, limit=12, M=None, N=None):
     and N given and the shape dispatched to the wide kernel (four row blocks per workgroup, so its good splits are
     larger): 1..32, never more than half of the group-tile columns."""
     nkb = K // 64
-    if M is not None and N is not None and b"wide" in (A.library().SpMM_KernelName(M, N, K, 1) or b""):
+    # from N = 256 on the kernel can depend on the split: the cost model's own split says which one a shape is for
+    if M is not None and N is not None and b"wide" in (
+            A.library().SpMM_KernelName(M, N, K, A.SpMM_SplitK_CostModel(M, N, K)) or b""):
         return [s for s in range(1, 33) if s <= max(1, nkb // 2)]
     return [s for s in range(1, limit + 1) if s <= max(1, nkb // 4)]
 
