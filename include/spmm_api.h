@@ -161,8 +161,8 @@ size_t SpMM_WorkspaceBytesBiasAct(int M, int N, int K, int Split_K);
  * SPMM_NOALLOC_SCRATCH_BYTES that the library itself holds on every GPU it runs on until the process ends.
  * Arguments and results are those of SpMM_SplitK_API (the same kernels run).  An explicit Split_K whose partial
  * sums (4*M*N*Split_K bytes for Split_K > 1) exceed the array prints a message and returns 1
- * (hipErrorInvalidValue) without launching anything.  With Split_K <= 0 the library's own choice gives way to the
- * largest split whose partial sums fit (an unsplit K needs none, so such a call always runs);
+ * (hipErrorInvalidValue) without launching anything.  With Split_K <= 0 the library's own choice, where its partial
+ * sums do not fit, gives way to a split whose partial sums do (an unsplit K needs none, so such a call always runs);
  * SpMM_SplitK_AutoNoAlloc reports that split.  The call makes no hipMalloc/hipFree; the first call on a
  * device looks up the array's device address once (make that call outside a graph capture).
  * All calls on one GPU share the array: calls that overlap in time on one GPU (different streams, or graphs

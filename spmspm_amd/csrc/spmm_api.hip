@@ -68,28 +68,37 @@ int auto_split_k_wide(int M, int N, int K)
     return best;
 }
 
-// Picks the K split from a small cost model (units: group tiles processed by the busiest CU), fitted to whole-call
-// times (main kernel + reduction, back to back on one stream) of ten OPT-like shapes at Split_K 1..20, where its
-// choice is within 4 % of the best measured split:
+constexpr int kMaxAutoSplit = 32; // the largest split the library chooses by itself
+
+// Split of a shape whose kernel goes with the split (spmm::kernel_by_split): the cheapest of 1..max_split, each with
+// the kernel the dispatch gives it.
+int auto_split_k_both(int M, int N, int K, int max_split)
+{
+    int    best   = 1;
+    double best_c = 1e30;
+    for (int sk = 1; sk <= max_split && sk <= kMaxAutoSplit && sk <= K / 64; ++sk) {
+        const double c = (spmm::use_wide_kernel(M, N, K, sk) ? spmm::main_wide_us(M, N, K, sk)
+                                                             : spmm::main_rows_us(M, N, K, sk)) +
+                         spmm::split_us(M, N, sk);
+        if (c < best_c - 1e-9) {
+            best_c = c;
+            best   = sk;
+        }
+    }
+    return best;
+}
+
+// The K split a call that leaves it to the library gets: from auto_split_k_both or auto_split_k_wide, and for the
+// shapes that run on the row-per-lane kernel at any split from a small cost model of its own (units: group tiles
+// processed by the busiest CU), fitted to whole-call times (main kernel + reduction, back to back on one stream) of
+// ten OPT-like shapes at Split_K 1..20, where its choice is within 4 % of the best measured split:
 //   work     ceil(workgroups / 256) turns of (tiles per workgroup + a fixed start-up/epilogue cost);
 //   fill     with fewer than two workgroups per CU the waves cannot hide each other's latencies;
 //   partials a split adds the reduction kernel, and every batch writes and re-reads an fp32 slab of M*N.
 int auto_split_k(int M, int N, int K)
 {
-    if (spmm::kernel_by_split(M, N, K)) { // split and kernel together
-        int    best   = 1;
-        double best_c = 1e30;
-        for (int sk = 1; sk <= 32 && sk <= K / 64; ++sk) {
-            const double c = (spmm::use_wide_kernel(M, N, K, sk) ? spmm::main_wide_us(M, N, K, sk)
-                                                                 : spmm::main_rows_us(M, N, K, sk)) +
-                             spmm::split_us(M, N, sk);
-            if (c < best_c - 1e-9) {
-                best_c = c;
-                best   = sk;
-            }
-        }
-        return best;
-    }
+    if (spmm::kernel_by_split(M, N, K))
+        return auto_split_k_both(M, N, K, kMaxAutoSplit);
     if (spmm::use_wide_kernel(M, N, K, 1))
         return auto_split_k_wide(M, N, K);
     const int    nkb  = K / 64;
@@ -500,6 +509,27 @@ void* scratch_address(hipError_t* err)
     return found;
 }
 
+// The library's own split, held to what the array fits (an unsplit K has no partial sums).  Where the kernel goes with
+// the split the search is run again among the splits that fit: the largest of them, taken unseen, can be one that only
+// the row-per-lane kernel runs, with every slab the array holds.  Whole calls at 60 % sparsity in us (Split_K):
+//   M x K, N          largest that fits / searched        M x K, N          largest that fits / searched
+//   1408x4416, 1408        63.7 (4) / 51.3 (1)            1344x13504, 512       67.5 (12) / 49.9 (10)
+//   3136x4416,  640        65.2 (4) / 50.9 (1)            1216x26880, 512      101.3 (13) / 70.9 (12)
+//   5440x5568,  384        75.6 (4) / 61.6 (1)            1408x11008, 640       77.2 (9)  / 50.8 (8)
+// On the other shapes the largest split that fits stays: auto_split_k_wide asked again prefers one workgroup to a CU,
+// which was better on ten of twelve shapes (5952x9792, N = 128: 43.9 / 41.5) and worse on two (21824x4672, N = 128:
+// 65.5 / 71.4).
+int noalloc_split_k(int M, int N, int K)
+{
+    const int    sk  = split_k_for(M, N, K);
+    const size_t fit = (size_t)SPMM_NOALLOC_SCRATCH_BYTES / (sizeof(float) * (size_t)M * (size_t)N);
+    if (sk <= 1 || (size_t)sk <= fit)
+        return sk;
+    if (fit < 2)
+        return 1;
+    return spmm::kernel_by_split(M, N, K) ? auto_split_k_both(M, N, K, (int)fit) : (int)fit;
+}
+
 } // namespace
 
 extern "C" int SpMM_SplitK_API_NoAlloc(hipStream_t stream, const void* values, const uint64_t* bitmaps,
@@ -507,14 +537,8 @@ extern "C" int SpMM_SplitK_API_NoAlloc(hipStream_t stream, const void* values, c
 {
     if (int e = check_shape(M, N, K))
         return refuse(e);
-    int          sk   = Split_K <= 0 ? split_k_for(M, N, K) : clamp_split_k(Split_K, K);
+    const int    sk   = Split_K <= 0 ? noalloc_split_k(M, N, K) : clamp_split_k(Split_K, K);
     const size_t slab = sizeof(float) * (size_t)M * (size_t)N;
-    if (Split_K <= 0 && sk > 1 && slab * (size_t)sk > (size_t)SPMM_NOALLOC_SCRATCH_BYTES) {
-        // the library's own choice gives way to the largest split whose partial sums fit; an unsplit K needs none
-        sk = (int)((size_t)SPMM_NOALLOC_SCRATCH_BYTES / slab);
-        if (sk < 2)
-            sk = 1;
-    }
     const size_t need = sk > 1 ? slab * (size_t)sk : 0;
     if (need > (size_t)SPMM_NOALLOC_SCRATCH_BYTES) {
         std::printf("MM_Sparse_API Error: M=%d N=%d Split_K=%d needs %zu bytes of partial sums; "
@@ -541,14 +565,7 @@ extern "C" int SpMM_SplitK_AutoNoAlloc(int M, int N, int K)
 {
     if (!supported_n(N) || M <= 0 || K <= 0 || M % 64 != 0 || K % 64 != 0)
         return 1;
-    int          sk   = split_k_for(M, N, K);
-    const size_t slab = sizeof(float) * (size_t)M * (size_t)N;
-    if (sk > 1 && slab * (size_t)sk > (size_t)SPMM_NOALLOC_SCRATCH_BYTES) {
-        sk = (int)((size_t)SPMM_NOALLOC_SCRATCH_BYTES / slab);
-        if (sk < 2)
-            sk = 1;
-    }
-    return sk;
+    return noalloc_split_k(M, N, K);
 }
 
 // ---- the six weight files -> device arrays (the consumer side of Our_GenSparseMatrixBinFile) -------------------

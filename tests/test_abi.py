@@ -293,6 +293,24 @@ def test_kernel_of_a_small_matrix_with_many_columns_follows_its_split(M, N, K, s
     assert own == 1 or 4 * M * N * own <= S.api.NOALLOC_SCRATCH_BYTES
 
 
+@pytest.mark.parametrize("M,N,K,good", [
+    (1408, 1408, 4416, {1}), (3136, 640, 4416, {1}), (5440, 384, 5568, {1, 3}), (2752, 1024, 2240, {1}),
+    (1344, 512, 13504, {10}), (1216, 512, 26880, {11, 12}), (1408, 640, 11008, {7, 8}), (640, 640, 25216, {16, 17}),
+])
+def test_no_alloc_split_is_searched_among_those_that_fit(M, N, K, good):
+    """Shapes whose own split needs more than the library's array holds.  `good`: the splits whose measured call is
+    within 10 % of the best that fits.  The largest that fits is none of them: it was 24 to 52 % slower."""
+    assert S.SpMM_SplitK_AutoNoAlloc(M, N, K) in good
+
+
+def test_no_alloc_split_fits_and_is_the_librarys_own_where_that_fits():
+    for M, N, K in [(512, 256, 512), (9344, 128, 5824), (28672, 2048, 7168), (640, 896, 9344), (4160, 384, 4928)]:
+        fit, own = S.api.NOALLOC_SCRATCH_BYTES // (4 * M * N), S.SpMM_SplitK_AutoNoAlloc(M, N, K)
+        assert own == 1 or own <= fit
+        if S.SpMM_SplitK_Auto(M, N, K) <= fit:
+            assert own == S.SpMM_SplitK_Auto(M, N, K)
+
+
 def test_row_count_limit_is_reported(capfd):
     """Row blocks are the z dimension of the launch grid: more than 65535 of them is refused before any launch."""
     L = S.library()
