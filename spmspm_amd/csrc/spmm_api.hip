@@ -77,9 +77,7 @@ int auto_split_k_both(int M, int N, int K, int max_split)
     int    best   = 1;
     double best_c = 1e30;
     for (int sk = 1; sk <= max_split && sk <= kMaxAutoSplit && sk <= K / 64; ++sk) {
-        const double c = (spmm::use_wide_kernel(M, N, K, sk) ? spmm::main_wide_us(M, N, K, sk)
-                                                             : spmm::main_rows_us(M, N, K, sk)) +
-                         spmm::split_us(M, N, sk);
+        const double c = spmm::call_us(M, N, K, sk, spmm::use_wide_kernel(M, N, K, sk));
         if (c < best_c - 1e-9) {
             best_c = c;
             best   = sk;
