@@ -777,6 +777,49 @@ def test_unsplit_tail_of_the_wide_kernel_equals_the_reduction(torch, variants_li
     assert np.array_equal(got[0], got[1])
 
 
+def test_gelu_is_the_nearest_half(torch, variants_lib):
+    """GELU of known sums (W the identity) in the wide kernel's tail and in the reduction.  An fp32 evaluation good to a
+    few 1e-7 gives the half nearest to the exact value but where that lies within this error of the middle between two
+    halves (spaced 2^-11 to 2^-10 of the value): in fewer than 0.4 % of the cases.  A sum 1 + tanh(u) that cancels for
+    negative x does not (2.8 %).  Infinities, signed zeros and NaN as 0.5 x (1 + tanh) gives them."""
+    import ctypes as C
+    M = K = 256
+    N = 128
+    rng = np.random.default_rng(5)
+    X = np.where(rng.random((N, K)) < 0.5, rng.uniform(-12, 12, (N, K)), rng.normal(0, 1.5, (N, K))).astype(np.float16)
+    dev = Device(torch, S.InitSparseMatrixA_bitmap(np.eye(M, dtype=np.float16)))
+    call = variants_lib.SpMM_SplitK_API_BiasAct
+    call.restype, call.argtypes = C.c_int, [C.c_void_p] * 6 + [C.c_int] * 3 + [C.c_void_p, C.c_int, C.c_void_p, C.c_int]
+
+    def gelu(x, variant, bias=None):
+        print(f"case gelu variant={variant} bias={bias is not None}", flush=True)
+        variants_lib.SpMM_Debug_SetKernelVariant(variant)
+        xd = torch.from_numpy(x.view(np.int16).copy()).to("cuda:0")
+        b = None if bias is None else torch.from_numpy(bias.view(np.int16).copy()).to("cuda:0")
+        out = torch.full((N, M), 0x7e00, dtype=torch.int16, device="cuda:0")
+        ws = torch.empty(4 * M * N, dtype=torch.uint8, device="cuda:0")
+        assert call(torch.cuda.current_stream().cuda_stream, dev.values.data_ptr(), dev.bitmaps.data_ptr(),
+                    dev.offsets.data_ptr(), xd.data_ptr(), out.data_ptr(), M, N, K, ws.data_ptr(), 1,
+                    None if b is None else b.data_ptr(), 2) == 0
+        torch.cuda.synchronize()
+        return out.cpu().numpy().view(np.float16)
+
+    x = X.astype(np.float64)
+    want = (0.5 * x * (1 + np.tanh(0.7978845608028654 * (x + 0.044715 * x ** 3)))).astype(np.float16)
+    special = np.zeros(M, np.float16)
+    special[:6] = [np.inf, -np.inf, np.nan, 65504.0, -65504.0, -0.0]
+    try:
+        for variant in (3, 4):
+            got = gelu(X, variant)
+            assert (got.view(np.uint16) != want.view(np.uint16)).mean() < 4e-3
+            assert np.abs(got.astype(np.float64) - want.astype(np.float64)).max() <= 2.0 ** -7  # one half's step below 16
+            s = gelu(np.zeros_like(X), variant, special)[0].astype(np.float32)
+            assert s[0] == np.inf and np.isnan(s[1]) and np.isnan(s[2]) and s[3] == 65504.0
+            assert (s[4:] == 0).all()
+    finally:
+        variants_lib.SpMM_Debug_SetKernelVariant(2)
+
+
 def test_bias_activation_errors_and_layer(torch, oracle, capfd):
     t = torch.zeros(64, dtype=torch.int16, device="cuda:0")
     assert S.SpMM_SplitK_API_BiasAct(None, t, t, t, t, t, 64, 16, 64, t, 1, None, 7) == S.api.HIP_ERROR_INVALID_VALUE
