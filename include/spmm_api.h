@@ -145,8 +145,9 @@ size_t SpMM_WorkspaceBytes(int M, int N, int K, int Split_K);
  * FasterTransformer layer (third_party/ft_spinfer.patch:766-768 and the unpatched FfnLayer code around it); no
  * such entry point exists in the reference's library.  `bias` is M fp16 values on the device, or NULL.
  * `activation`: 0 none, 1 ReLU, 2 GELU in its tanh form 0.5*x*(1 + tanh(0.79788456*(x + 0.044715*x^3))).
- * The partial sums always pass through `workspace` (fp32), which must hold
- * SpMM_WorkspaceBytesBiasAct(M, N, K, Split_K) bytes = 4*M*N*max(Split_K, 1), also for an unsplit K.
+ * `workspace` must hold SpMM_WorkspaceBytesBiasAct(M, N, K, Split_K) bytes = 4*M*N*max(Split_K, 1) and is refused
+ * when NULL, for an unsplit K too.  The fp32 partial sums of a split K pass through it; an unsplit K has none, its
+ * kernel applies bias and activation itself and leaves the workspace as it was.
  * Other arguments, Split_K <= 0 and return values as for SpMM_SplitK_API; an unknown activation returns 1.
  */
 int SpMM_SplitK_API_BiasAct(hipStream_t stream, const void* values, const uint64_t* bitmaps, const int* offsets,
@@ -297,8 +298,10 @@ int SpMM_ShaderClockProbe(hipStream_t stream, unsigned long long* ticks_d, int s
  * Name of the main kernel a call of SpMM_SplitK_API, SpMM_SplitK_API_Sized or SpMM_SplitK_API_NoAlloc with these
  * dimensions dispatches, as a profiler prints it, e.g. "spmm::spmm_bitmap_rows<1, true>" (second template argument:
  * fp32 partial sums to the workspace, which these three entry points use whenever K is split).  It does not hold
- * for SpMM_SplitK_API_bitmap_v3 (fp16 partial sums: "false" for every split) or SpMM_SplitK_API_BiasAct (one fp32
- * slab even for an unsplit K: "true" for every split).  Split_K <= 0 asks for the library's own split.  Reporting aid for benchmarks that key profiler records by kernel; no
+ * for SpMM_SplitK_API_bitmap_v3 (fp16 partial sums: "false" for every split) or for SpMM_SplitK_API_BiasAct with a
+ * bias or an activation and an unsplit K ("spmm::spmm_bitmap_row_tail<1>" in the place of
+ * "spmm::spmm_bitmap_rows<1, false>", "spmm::spmm_bitmap_wide_tail<8>" in that of "spmm::spmm_bitmap_wide<8, false>").
+ * Split_K <= 0 asks for the library's own split.  Reporting aid for benchmarks that key profiler records by kernel; no
  * reference counterpart.  The string belongs to the library and is valid until the thread's next call of this
  * function; NULL for dimensions the SpMM calls refuse.
  */

@@ -301,7 +301,7 @@ int run(hipStream_t stream, const void* values, const uint64_t* bitmaps, const i
     hipError_t err = spmm::launch_spmm(stream, static_cast<const __half*>(values), bitmaps, offsets,
                                        static_cast<const __half*>(X), static_cast<__half*>(C), M, N, K, workspace,
                                        split_k, fp32_partials, before, after, epilogue, bias, act);
-    if (err != hipSuccess || spmm::main_kernel_finishes(M, N, K, split_k, epilogue))
+    if (err != hipSuccess || spmm::main_kernel_finishes(split_k, epilogue))
         return (int)err;
     return (int)spmm::launch_reduction(stream, static_cast<__half*>(C), workspace, M, N, split_k, fp32_partials, bias,
                                        act);

@@ -25,3 +25,17 @@ def test_main_kernel_occupancy_budget():
             assert r["vgpr"] <= limit[key], (name, r)
             seen += 1
     assert seen == 6
+
+
+def test_wide_kernels_and_tails_occupancy_budget():
+    """Two workgroups of the wide kernel to a CU: at most 256 registers, tail or not.  The unsplit tails of the row-per-lane
+    kernel keep the budget of the kernels they stand beside."""
+    res = build.kernel_resources("spmm_api.hip")
+    limit = {"row_tailILi1E": 128, "row_tailILi2E": 168, "row_tailILi4E": 256, "spmm_bitmap_wide": 256}
+    seen = 0
+    for name, r in res.items():
+        for key in limit:
+            if key in name:
+                assert r["vgpr"] <= limit[key], (name, r)
+                seen += 1
+    assert seen == 3 + 6

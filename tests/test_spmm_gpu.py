@@ -748,8 +748,9 @@ def test_bias_activation_entry_point(torch, oracle, M, K, N, s, sk, act, with_bi
 @pytest.mark.parametrize("act", [0, 1, 2])
 @pytest.mark.parametrize("with_bias", [False, True])
 def test_unsplit_tail_of_the_wide_kernel_equals_the_reduction(torch, variants_lib, M, K, N, act, with_bias):
-    """At Split_K = 1 the wide kernel applies bias and activation to its accumulators, the row-per-lane kernel leaves
-    them to the reduction.  With exact sums (small integers) both round the same fp32 value once: equal bit for bit."""
+    """At Split_K = 1 the wide kernel applies bias and activation to its accumulators and the row-per-lane kernel to the
+    sum of its four waves; at Split_K = 2 the reduction does.  With exact sums (small integers) all round the same fp32
+    value once: equal bit for bit."""
     import ctypes as C
     rng = np.random.default_rng(M + N)
     W, X = _small_integer_problem(rng, M, K, N, 0.5)
@@ -762,23 +763,23 @@ def test_unsplit_tail_of_the_wide_kernel_equals_the_reduction(torch, variants_li
     call.restype, call.argtypes = C.c_int, [C.c_void_p] * 6 + [C.c_int] * 3 + [C.c_void_p, C.c_int, C.c_void_p, C.c_int]
     got = []
     try:
-        for variant in (3, 4):
-            print(f"case tail M={M} K={K} N={N} act={act} bias={with_bias} variant={variant}", flush=True)
+        for variant, split_k in ((3, 1), (4, 1), (3, 2 if K > 64 else 1)):
+            print(f"case tail M={M} K={K} N={N} act={act} bias={with_bias} variant={variant} Split_K={split_k}", flush=True)
             variants_lib.SpMM_Debug_SetKernelVariant(variant)
             out = torch.full((N, M), 0x7e00, dtype=torch.int16, device="cuda:0")
-            ws = torch.empty(4 * M * N, dtype=torch.uint8, device="cuda:0")
+            ws = torch.empty(4 * M * N * split_k, dtype=torch.uint8, device="cuda:0")
             assert call(torch.cuda.current_stream().cuda_stream, dev.values.data_ptr(), dev.bitmaps.data_ptr(),
-                        dev.offsets.data_ptr(), x.data_ptr(), out.data_ptr(), M, N, K, ws.data_ptr(), 1,
+                        dev.offsets.data_ptr(), x.data_ptr(), out.data_ptr(), M, N, K, ws.data_ptr(), split_k,
                         b.data_ptr() if with_bias else None, act) == 0
             torch.cuda.synchronize()
             got.append(out.cpu().numpy())
     finally:
         variants_lib.SpMM_Debug_SetKernelVariant(2)
-    assert np.array_equal(got[0], got[1])
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
 
 
 def test_gelu_is_the_nearest_half(torch, variants_lib):
-    """GELU of known sums (W the identity) in the wide kernel's tail and in the reduction.  An fp32 evaluation good to a
+    """GELU of known sums (W the identity) in the tails of both kernels and in the reduction.  An fp32 evaluation good to a
     few 1e-7 gives the half nearest to the exact value but where that lies within this error of the middle between two
     halves (spaced 2^-11 to 2^-10 of the value): in fewer than 0.4 % of the cases.  A sum 1 + tanh(u) that cancels for
     negative x does not (2.8 %).  Infinities, signed zeros and NaN as 0.5 x (1 + tanh) gives them."""
@@ -791,15 +792,15 @@ def test_gelu_is_the_nearest_half(torch, variants_lib):
     call = variants_lib.SpMM_SplitK_API_BiasAct
     call.restype, call.argtypes = C.c_int, [C.c_void_p] * 6 + [C.c_int] * 3 + [C.c_void_p, C.c_int, C.c_void_p, C.c_int]
 
-    def gelu(x, variant, bias=None):
-        print(f"case gelu variant={variant} bias={bias is not None}", flush=True)
+    def gelu(x, variant, split_k, bias=None):
+        print(f"case gelu variant={variant} Split_K={split_k} bias={bias is not None}", flush=True)
         variants_lib.SpMM_Debug_SetKernelVariant(variant)
         xd = torch.from_numpy(x.view(np.int16).copy()).to("cuda:0")
         b = None if bias is None else torch.from_numpy(bias.view(np.int16).copy()).to("cuda:0")
         out = torch.full((N, M), 0x7e00, dtype=torch.int16, device="cuda:0")
-        ws = torch.empty(4 * M * N, dtype=torch.uint8, device="cuda:0")
+        ws = torch.empty(4 * M * N * split_k, dtype=torch.uint8, device="cuda:0")
         assert call(torch.cuda.current_stream().cuda_stream, dev.values.data_ptr(), dev.bitmaps.data_ptr(),
-                    dev.offsets.data_ptr(), xd.data_ptr(), out.data_ptr(), M, N, K, ws.data_ptr(), 1,
+                    dev.offsets.data_ptr(), xd.data_ptr(), out.data_ptr(), M, N, K, ws.data_ptr(), split_k,
                     None if b is None else b.data_ptr(), 2) == 0
         torch.cuda.synchronize()
         return out.cpu().numpy().view(np.float16)
@@ -809,15 +810,72 @@ def test_gelu_is_the_nearest_half(torch, variants_lib):
     special = np.zeros(M, np.float16)
     special[:6] = [np.inf, -np.inf, np.nan, 65504.0, -65504.0, -0.0]
     try:
-        for variant in (3, 4):
-            got = gelu(X, variant)
+        for variant, split_k in ((3, 1), (4, 1), (3, 2)):
+            got = gelu(X, variant, split_k)
             assert (got.view(np.uint16) != want.view(np.uint16)).mean() < 4e-3
             assert np.abs(got.astype(np.float64) - want.astype(np.float64)).max() <= 2.0 ** -7  # one half's step below 16
-            s = gelu(np.zeros_like(X), variant, special)[0].astype(np.float32)
+            s = gelu(np.zeros_like(X), variant, split_k, special)[0].astype(np.float32)
             assert s[0] == np.inf and np.isnan(s[1]) and np.isnan(s[2]) and s[3] == 65504.0
             assert (s[4:] == 0).all()
     finally:
         variants_lib.SpMM_Debug_SetKernelVariant(2)
+
+
+@pytest.mark.parametrize("M,K,N,kernel", [
+    (192, 320, 8, "rows<1"), (64, 192, 16, "rows<1"), (320, 128, 32, "rows<2"), (192, 448, 64, "rows<4"),
+    (320, 640, 384, "rows<4"), (3648, 320, 1152, "wide<8"),
+])
+def test_unsplit_bias_and_activation_need_no_partial_sums(torch, M, K, N, kernel):
+    """The shipped library's own dispatch: whichever kernel an unsplit call with bias or activation runs on applies
+    them itself.  Against float64; the workspace is left as it was; and with exact sums (small integers) the result is
+    bit for bit that of a split call, whose sums go through the reduction."""
+    assert kernel in S.library().SpMM_KernelName(M, N, K, 1).decode()
+    rng = np.random.default_rng(M + N)
+    bias = rng.uniform(-2, 2, M).astype(np.float16)
+    bias[[0, 63, M - 1]] = [1.0, -1.0, -0.0]
+    b = torch.from_numpy(bias.view(np.int16).copy()).to("cuda:0")
+
+    def call(dev, x, split_k, with_bias, act):
+        print(f"case M={M} K={K} N={N} Split_K={split_k} bias={with_bias} act={act}", flush=True)
+        out = torch.full((N, M), 0x7e00, dtype=torch.int16, device="cuda:0")
+        ws = torch.full((M * N * split_k,), 0x7fc00000, dtype=torch.int32, device="cuda:0")  # NaN
+        assert S.SpMM_SplitK_API_BiasAct(None, dev.values, dev.bitmaps, dev.offsets, x, out, M, N, K, ws, split_k,
+                                         b if with_bias else None, act) == 0
+        torch.cuda.synchronize()
+        assert split_k > 1 or bool((ws == 0x7fc00000).all())
+        return out.cpu().numpy().view(np.float16)
+
+    W, X = make_weight(M, K, 0.6, seed=M), make_activations(K, N, seed=K)
+    dev, x = Device(torch, S.InitSparseMatrixA_bitmap(W)), torch.from_numpy(X.view(np.int16).copy()).to("cuda:0")
+    sums = X.astype(np.float64) @ W.astype(np.float64).T
+    for with_bias, act in ((True, 0), (False, 1), (True, 1), (True, 2), (False, 2)):
+        pre = sums + bias.astype(np.float64) if with_bias else sums
+        want = pre if act == 0 else (np.maximum(pre, 0) if act == 1
+                                     else 0.5 * pre * (1 + np.tanh(0.7978845608028654 * (pre + 0.044715 * pre ** 3))))
+        assert_spmm_close(call(dev, x, 1, with_bias, act), want, f"bias={with_bias} act={act}")
+
+    W, X = _small_integer_problem(rng, M, K, N, 0.3)
+    dev, x = Device(torch, S.InitSparseMatrixA_bitmap(W)), torch.from_numpy(X.view(np.int16).copy()).to("cuda:0")
+    for with_bias, act in ((True, 0), (False, 1), (True, 1), (True, 2), (False, 2)):
+        assert np.array_equal(call(dev, x, 1, with_bias, act).view(np.uint16),
+                              call(dev, x, 2, with_bias, act).view(np.uint16)), (with_bias, act)
+
+
+@pytest.mark.parametrize("M,K,N,entry,split_k,kernel", [
+    (3648, 320, 1152, "api", 0, "wide<8"), (1216, 192, 1152, "api", 3, "wide<8"), (1216, 192, 1152, "v3", 3, "wide<8"),
+    (1216, 192, 1152, "api", 2, "rows<4"), (2752, 128, 768, "v3", 2, "wide<8"), (4160, 4928, 384, "api", 0, "wide<8"),
+    (4160, 4928, 384, "api", 5, "wide<8"), (4160, 4928, 384, "v3", 2, "rows<4"), (704, 3584, 768, "api", 0, "rows<4"),
+])
+def test_kernel_chosen_by_the_split_is_exact(torch, M, K, N, entry, split_k, kernel):
+    """From N = 256 on a small matrix's kernel goes with the split, the library's or the caller's: the shipped library on
+    both sides of that rule, row blocks that do not fill a quad of the wide kernel among them.  Small integers: every
+    partial sum is exact, in fp16 too, and so is the result but for its one rounding."""
+    assert kernel in S.library().SpMM_KernelName(M, N, K, split_k).decode()
+    W, X = _small_integer_problem(np.random.default_rng(M + K), M, K, N, 0.4)
+    want = (X.astype(np.float64) @ W.astype(np.float64).T).astype(np.float16)
+    dev = Device(torch, S.InitSparseMatrixA_bitmap(W))
+    print(f"case M={M} K={K} N={N} {entry} Split_K={split_k}", flush=True)
+    assert np.array_equal(dev.spmm(X, split_k, entry).view(np.uint16), (want + np.float16(0)).view(np.uint16))
 
 
 def test_bias_activation_errors_and_layer(torch, oracle, capfd):
